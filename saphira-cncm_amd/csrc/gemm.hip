@@ -1329,6 +1329,8 @@ __device__ __forceinline__ void gemm_big_body(const GemmArgs &pa) {
             if (i0 + tid < p.Mo) p.db[i] = old + (0.0f + (float)d);
         }
     }
+    // (heads, an odd number of them: the last tile column's upper waves have no head)
+    if (SEL == SEL_HEADS && j0 + wn * 64 >= pa.No) return;
     g_epilogue_big<EPI, !AKC, !BKC>(p, tot, i0, j0, tid);
 }
 

@@ -247,3 +247,34 @@ def test_capture_takes_the_fp32_kernel():
         assert bits_equal(got, y.numpy())
     hip.hipGraphExecDestroy(ex)
     hip.hipGraphDestroy(graph)
+
+
+@pytest.mark.parametrize("mode", [64, 128, 1064, 1128])
+@pytest.mark.parametrize("B,T,H,M", [(3, 64, 3, 128), (1, 128, 3, 68), (1, 192, 1, 64), (2, 64, 2, 256)])
+def test_head_gradient_at_the_last_tiles(mode, B, T, H, M):
+    """dX added into a head-major gradient where the outputs end inside a
+    128 x 128 tile (an odd number of heads, an odd number of 64-row blocks):
+    the waves past the end belong to no head and no sequence and must not touch
+    memory; the guard floats around the gradient keep their bits."""
+    rng = np.random.default_rng(29)
+    lib, K, rows, guard = ncmhip.load(), 64 * H, B * T, 256
+    dy, W = rng.integers(-3, 4, (rows, M)).astype(np.float32), rng.integers(-3, 4, (M, K)).astype(np.float32)
+    old = rng.integers(-9, 10, (B, H, T, 64)).astype(np.float32)
+    prod = (dy @ W).reshape(B, T, H, 64).transpose(0, 2, 1, 3)
+    fn = lib.ncm_linear_bwd_heads
+    vp, ci = ctypes.c_void_p, ctypes.c_int
+    fn.restype, fn.argtypes = None, [vp, vp, vp, vp, ci, vp, vp, ci, ci, ci, ci]
+    Wd, dyd = D.from_numpy(W), D.from_numpy(dy)
+    print(f"[gpu] heads dX {B}x{T} x {H} heads, M {M}, mode {mode}", flush=True)
+    lib.ncm_hip_set_gemm_tiles(mode)
+    try:
+        for beta in (0, 1):
+            edge = np.full(guard, 7.5, np.float32)
+            buf = D.from_numpy(np.concatenate([edge, old.reshape(-1), edge]))
+            fn(None, Wd.ptr, dyd.ptr, buf.ptr + 4 * guard, beta, None, None, B, T, M, H)
+            ncmhip.check()
+            got = buf.numpy()
+            assert bits_equal(got[:guard], edge) and bits_equal(got[-guard:], edge)
+            assert bits_equal(got[guard:-guard].reshape(old.shape), old * beta + prod + np.float32(0.0))
+    finally:
+        lib.ncm_hip_set_gemm_tiles(0)
