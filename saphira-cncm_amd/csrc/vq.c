@@ -135,10 +135,10 @@ static int vq_fits16(int V, int D) {
 
 /* The screens that start on the fp16 matrix cores: packs the rows (after `u`,
  * the last level's update, when given) and codewords, screens them in fp16 and
- * the rows then undecided in FP32.  1: done; 0: not for this shape, or its
- * workspace is not to be had (under stream capture, for one), and nothing was
- * launched; < 0: an error. */
-static int vq_screen16(VqArgs p, const VqUpdate *u, unsigned *counters) {
+ * the rows then undecided in FP32.  Returns 0 or an error code; *done is set
+ * where the screens were launched, and stays 0 where this shape is not for
+ * them or their workspace is not to be had (under stream capture, for one). */
+static int vq_screen16(VqArgs p, const VqUpdate *u, unsigned *counters, int *done) {
     if (!vq_fits16(p.V, p.D)) return 0;
     int ks = p.D <= 64 ? 2 : p.D <= 128 ? 4 : 8, rc;
     const size_t wgs = ((size_t)p.rows + VQR - 1) / VQR, tiles = ((size_t)p.V + 63) / 64;
@@ -194,7 +194,8 @@ static int vq_screen16(VqArgs p, const VqUpdate *u, unsigned *counters) {
     if ((rc = ncm_launch_named(vec ? "vq_argmin_list_v" : "vq_argmin_list_s",
                                (unsigned)(items < VQ_PARTS ? items : VQ_PARTS), 1, 1, 256, al)))
         return rc;
-    return 1;
+    *done = 1;
+    return 0;
 }
 
 /* codes of `rows` rows of X against E, written at idx[(row/L)*total + off + row%L];
@@ -203,14 +204,14 @@ static int vq_search(const float *X, const float *E, int *idx, int rows, int V, 
                      int total, int off, unsigned char *scratch, const VqUpdate *u) {
     VqScratch s;
     if (vq_scratch(&s, rows, V, scratch)) return NCM_E_OOM;
-    int rc;
+    int rc, done = 0;
     unsigned *cmax = s.counters + 1;
     int vec = (D % 4 == 0) && is_aligned16(X) && is_aligned16(E);
     VqArgs p = {X, E, s.cn, s.xn, cmax, idx, s.flags, (int *)s.counters,
                 s.pairs, (int *)s.counters + 2, s.keys, s.done, rows, V, D, L, total, off,
                 NULL, NULL, NULL, NULL, NULL, 0, NULL, NULL, NULL, NULL};
-    if ((rc = scratch ? 0 : vq_screen16(p, u, s.counters)) < 0) return rc;
-    if (!rc) {
+    if (!scratch && (rc = vq_screen16(p, u, s.counters, &done))) return rc;
+    if (!done) {
         if (u && (rc = vq_residual(u, idx, rows, D, L, total))) return rc;
         void *a0[] = {&s.counters};
         if ((rc = ncm_launch_named("vq_init", 1, 1, 1, 64, a0))) return rc;
