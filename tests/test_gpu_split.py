@@ -278,3 +278,47 @@ def test_head_gradient_at_the_last_tiles(mode, B, T, H, M):
             assert bits_equal(got[guard:-guard].reshape(old.shape), old * beta + prod + np.float32(0.0))
     finally:
         lib.ncm_hip_set_gemm_tiles(0)
+
+
+@pytest.mark.parametrize("M,N,K,offset", [(512, 4864, 896, 0), (2048, 1152, 896, 0), (600, 770, 515, 1)])
+def test_capture_of_split_reductions(M, N, K, offset):
+    """Calls whose FP32 plans cut the reduction (partial tiles in a workspace,
+    bias sums in another): recorded right after the same calls ran eagerly on
+    the split-operand kernels, and replayed on new inputs."""
+    rng = np.random.default_rng(31)
+    lib, hip = ncmhip.load(), ctypes.CDLL("libamdhip64.so")
+
+    def put(shape):
+        return D.from_numpy(np.zeros(int(np.prod(shape)) + offset, np.float32))
+
+    def fill(buf, a):
+        buf.upload(np.concatenate([np.zeros(offset, np.float32), a.reshape(-1)]))
+    x, W, dy, y, dx, dW, db = (put(s) for s in ((M, K), (N, K), (M, N), (M, N), (M, K), (N, K), (N,)))
+    p = [b.ptr + 4 * offset for b in (x, W, dy, y, dx, dW, db)]
+    if offset == 0:
+        assert ncmhip.linear_plan("fwd", M, N, K)[1] > 1
+    assert ncmhip.linear_route("fwd", M, N, K)[0].startswith("split_")
+
+    def step():
+        ncmhip.linear_fwd(p[0], p[1], None, p[3], M, N, K)
+        ncmhip.linear_bwd(p[0], p[1], p[2], p[4], p[5], p[6], M, N, K)
+    step()
+    ncmhip.sync()
+    stream, graph, ex = ctypes.c_void_p(ncmhip.stream()), ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamBeginCapture(stream, 2) == 0
+    step()
+    assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(3):
+        a = [rng.integers(-3, 4, s).astype(np.float32) for s in ((M, K), (N, K), (M, N))]
+        for b, v in zip((x, W, dy), a):
+            fill(b, v)
+        for b, s in ((dx, (M, K)), (dW, (N, K)), (db, (N,))):
+            fill(b, np.zeros(s, np.float32))
+        assert hip.hipGraphLaunch(ex, stream) == 0
+        for b, want in zip((y, dx, dW, db), exact(*a)):
+            assert bits_equal(b.numpy()[offset:].reshape(want.shape), want.astype(np.float32))
+        step()   # the eager calls between the replays
+        ncmhip.sync()
+    hip.hipGraphExecDestroy(ex)
+    hip.hipGraphDestroy(graph)

@@ -1,7 +1,8 @@
 """What the host code launches, without a device: the library runs in a child
 process on stand-ins for the HIP calls (tests/c/fake_hip.c) that log them.
 A launch that fails ends its call: the kernels after it would work on what it
-should have written."""
+should have written.  A call that is recorded into a graph after the same call
+ran eagerly allocates, frees and waits for nothing: that would end the capture."""
 import json
 import os
 import subprocess
@@ -81,3 +82,12 @@ def test_nothing_is_launched_after_a_failed_launch(host, name, args):
     for n, r in enumerate(host(steps)):
         assert (r["error"] != 0) == (n > 0)
         assert launches(r) == (whole[:n] if n else whole)
+
+
+@pytest.mark.parametrize("name,args", CALLS + [("linear_fwd", (2048, 1152, 896)), ("linear_bwd", (4096, 768, 2304)),
+                                               ("linear_bwd", (4096, 771, 2301)), ("linear_bwd", (4096, 768, 2304, 4))])
+def test_capture_after_an_eager_call(host, name, args):
+    eager, captured = host([(name, args), (name, args, 0, 1)])
+    assert not eager["error"] and not captured["error"] and launches(captured)
+    assert not {"hipMalloc", "hipFree", "hipStreamSynchronize"} & set(captured["log"])
+    assert not any(w.startswith(("split_", "vq_screen16", "vq_pack")) for w in captured["log"])
