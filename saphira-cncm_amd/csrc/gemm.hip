@@ -94,11 +94,12 @@ struct GemmArgs {
     // [B][n3[part] / 64][T][64]; hm_T = T, a multiple of 64
     int hm_T;
     // split-operand kernels (gemm_split.h): the packed operands, their scales
-    // and panel counts, and how A and B themselves are stored (1: k-contiguous)
+    // and panel counts, and how A and B themselves are stored (1: k-contiguous;
+    // vec: and K and all rows are in 16-byte units)
     const char *Ap, *Bp;
     const float *As, *Bs;
     int panels_a, panels_b;
-    int a_kc, b_kc;
+    int a_kc, b_kc, a_vec, b_vec;
 };
 
 // SEL_HEADS: the tile at (i0, j0) lies in one head of one part and, T being a

@@ -322,3 +322,95 @@ def test_capture_of_split_reductions(M, N, K, offset):
         ncmhip.sync()
     hip.hipGraphExecDestroy(ex)
     hip.hipGraphDestroy(graph)
+
+
+def _spread(rng, M, K, N, kind, e):
+    """x, W, dy whose products are ordinary while values 2^e apart lie in one
+    scale group of 128 (along the features for y and dx, the rows for dW)."""
+    x, dy = (rng.standard_normal(s).astype(np.float32) for s in ((M, K), (M, N)))
+    W = (rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32)
+    if kind == "units":       # features (and outputs, and rows) of different units, weights that make up for them
+        f, o, r = (rng.integers(-e // 2, e // 2 + 1, (1, n)) for n in (K, N, M))
+        x, W, dy = np.ldexp(x, f + r.T), np.ldexp(W, -f + o.T), np.ldexp(dy, -o - r.T)
+    elif kind == "outlier":   # a large value where the other operand is zero
+        x[:, 5::97] *= 2.0 ** e
+        W[:, 5::97] = 0.0
+        W[3::70] = 0.0
+        dy[:, 3::70] *= 2.0 ** e
+        x[7::90] = 0.0
+        dy[7::90] *= 2.0 ** e
+    elif kind == "reader":    # the same, but one output and one feature read the large value
+        x[:, 5] *= 2.0 ** e
+        W[:, 5] = 0.0
+        W[-1, 5] = 1.0
+        dy[4] *= 2.0 ** e
+        x[4] = 0.0
+        x[4, -1] = 1.0
+    else:                     # tiny values beside ordinary ones, whole columns and rows of them
+        x[:, ::3] *= 2.0 ** -e
+        W[::3] *= 2.0 ** -e
+        dy[1::3] *= 2.0 ** -e
+        x[:, 1::3][rng.random(x[:, 1::3].shape) < 0.5] = 0.0
+    return tuple(np.asarray(a, np.float32) for a in (x, W, dy))
+
+
+@pytest.mark.parametrize("kind", ["units", "outlier", "reader", "tiny"])
+@pytest.mark.parametrize("e", [14, 20, 24, 30, 40, 60])
+@pytest.mark.parametrize("M,K,N", [(256, 384, 192), (131, 301, 141), (140, 100, 70)])
+def test_values_far_apart_in_a_group(tiles, M, K, N, e, kind):
+    """Two fp16 values hold a value to 2^-21 of itself down to 2^-19 of its
+    group's largest: outputs that depend on smaller ones are summed again in
+    FP32.  Element by element against sum |a b|, in float64: 2^-21 for each
+    factor, 2^-22 for the dropped l.l, 2^-22 that may be lost before an output is
+    summed again, and one rounding per MFMA and group sum."""
+    x, W, dy = _spread(np.random.default_rng(37 + e), M, K, N, kind, e)
+    got = run(x, W, dy)
+    sizes = exact(*[np.abs(v) for v in (x, W, dy)])
+    for g, want, size, red in zip(got, exact(x, W, dy), sizes, (K, N, M, M)):
+        groups = -(-red // 128)
+        bound = (6 * 2.0 ** -22 + (12 + groups + 2) * 2.0 ** -23) * size
+        assert np.all(np.abs(g - want) <= bound), (np.max(np.abs(g - want) / (size + 1e-300)) * 2.0 ** 23, groups)
+
+
+def test_units_of_features_in_every_form():
+    """Features of different units through the default routes: q | k | v side
+    by side, the gated unit and a cut reduction."""
+    rng = np.random.default_rng(41)
+    lib = ncmhip.load()
+    M, K, ns = 520, 768, (192, 64, 128)
+    f = rng.integers(-18, 19, (1, K))
+    x = np.ldexp(rng.standard_normal((M, K)), f).astype(np.float32)
+    Ws = [np.ldexp(rng.standard_normal((n, K)) / np.sqrt(K), -f).astype(np.float32) for n in ns]
+
+    def close(got, x, W, slack=1.0):
+        want, size = x.astype(np.float64) @ W.astype(np.float64).T, np.abs(x).astype(np.float64) @ np.abs(W).T
+        assert np.all(np.abs(got - want) <= slack * (6 * 2.0 ** -22 + (12 + 6 + 2) * 2.0 ** -23) * size)
+    xd, Wd, yd = D.from_numpy(x), [D.from_numpy(W) for W in Ws], [D.empty((M, n)) for n in ns]
+    P3 = ctypes.c_void_p * 3
+    fn = lib.ncm_linear_fwd3
+    fn.restype, fn.argtypes = None, [ctypes.c_void_p, P3, P3, P3, ctypes.c_int * 3, ctypes.c_int64, ctypes.c_int]
+    for mode in (1064, 1128):
+        lib.ncm_hip_set_gemm_tiles(mode)
+        fn(xd.ptr, P3(*[w.ptr for w in Wd]), P3(None, None, None), P3(*[y.ptr for y in yd]), (ctypes.c_int * 3)(*ns),
+           M, K)
+        ncmhip.check()
+        for y, W in zip(yd, Ws):
+            close(y.numpy(), x, W)
+    n = 150   # the gated unit without an activation: the product of two sums, each within its bound
+    Wg, Wu = (np.ldexp(rng.standard_normal((n, K)) / np.sqrt(K), -f).astype(np.float32) for _ in range(2))
+    o, gd, ud = D.empty((M, n)), D.from_numpy(Wg), D.from_numpy(Wu)
+    lib.linear_fwd_gated(xd.ptr, gd.ptr, None, ud.ptr, None, o.ptr, M, n, K, 0)
+    ncmhip.check()
+    lib.ncm_hip_set_gemm_tiles(0)
+    a, b = (x.astype(np.float64) @ w.astype(np.float64).T for w in (Wg, Wu))
+    sa, sb = (np.abs(x).astype(np.float64) @ np.abs(w).T for w in (Wg, Wu))
+    c = 6 * 2.0 ** -22 + (12 + 6 + 2) * 2.0 ** -23
+    assert np.all(np.abs(o.numpy() - a * b) <= c * (sa * np.abs(b) + sb * np.abs(a)) + c * c * sa * sb +
+                  2.0 ** -23 * np.abs(a * b))
+    xk, Wk = np.tile(x[:40], (1, 4)), np.tile(Ws[1], (1, 4))   # K = 3072, few tiles
+    lib.ncm_hip_set_gemm_tiles(1064)
+    assert ncmhip.linear_route("fwd", 40, 64, 3072)[1] > 1
+    y = D.empty((40, 64))
+    ncmhip.linear_fwd(D.from_numpy(xk), D.from_numpy(Wk), None, y, 40, 64, 3072)
+    lib.ncm_hip_set_gemm_tiles(0)
+    close(y.numpy(), xk, Wk, 2.0)
