@@ -342,7 +342,9 @@ static void sdpa_any_bm(const char *fn, const float *q, const float *k, const fl
         if (!stats && sdpa_split(q, k, v, mask, mask_bs, out, B, Hq, Hkv, Tq, Tkv, scale, causal, merged) <= 0)
             return;
         void *a[] = {&q, &k, &v, &mask, &out, &Hq, &Hkv, &Tq, &Tkv, &scale, &causal, &merged, &stats, &mask_bs};
-        ncm_launch_named(Tkv > 64 ? "sdpa16_hd64" : "sdpa_hd64", (unsigned)Hq, (unsigned)B, (unsigned)((Tq + 63) / 64), 256, a);
+        /* (up to two tiles of keys do not pay for the splitting) */
+        ncm_launch_named(Tkv > 128 ? "sdpa16_hd64" : "sdpa_hd64", (unsigned)Hq, (unsigned)B,
+                         (unsigned)((Tq + 63) / 64), 256, a);
     } else if (stats) {
         ncm_fail(NCM_E_ARG, "%s: row statistics need hd = 64 and 16-byte aligned operands", fn);
     } else {

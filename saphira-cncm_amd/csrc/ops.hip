@@ -639,10 +639,11 @@ __device__ __forceinline__ void sdpa_tile(const float *q, const float *k, const 
                        part_o, part_ml, mask_bs, sK, sV);
 }
 
-// sdpa_hd64 on the 16-bit matrix cores, for more than one tile of keys.  With
-// one tile nothing covers the splitting: 16 queries x 16 keys x 4 heads 6.2
-// against 5.8 us, 64 x 4 heads x 33 x 33 7.1 against 6.6; from two tiles on it
-// is even (8 x 4 x 81 x 81 9.7) or ahead.
+// sdpa_hd64 on the 16-bit matrix cores, for more than two tiles of keys.  With
+// one or two little covers the splitting (us, against sdpa_hd64's): 8 x 4 heads x
+// 81 x 81 11.2 : 9.7, 64 x 4 x 81 x 81 15.6 : 15.3, 128 x 4 x 100 x 100 causal
+// 24.0 : 21.5, 64 x 4 x 128 x 128 15.7 : 16.3; with three it is ahead: 64 x 4 x
+// 160 x 160 25.0 : 27.4, 32 x 12 x 192 x 192 causal 29.5 : 35.5.
 extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 sdpa16_hd64(const float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ v,
           const float *__restrict__ mask, float *__restrict__ out, int Hq, int Hkv, int Tq, int Tkv,

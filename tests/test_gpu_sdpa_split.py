@@ -101,3 +101,78 @@ def test_nonfinite():
         fin = np.isfinite(want)
         assert np.array_equal(np.isfinite(got), fin) and np.array_equal(np.isnan(got), np.isnan(want))
         assert rel(got[fin], want[fin]) < 1e-6
+
+
+def close(got, want, q, k, v, causal, mask=None):
+    """Element by element, in float64, against sum p |v| / sum p: a score is off
+    by sum |q k| / 8 times the 2^-21 of its pairs' representation (2 x 2^-23, l.l
+    2^-22) and some ten roundings of the sums (10 x 2^-24), and by 2^-23 of the
+    larger of 1 and the scores that the bound lets pass; p and V by as much of
+    themselves, their sum by 2^-21 and its roundings, one a tile."""
+    size = exact(q, k, np.abs(v), causal, mask)
+    g = q.shape[1] // k.shape[1]
+    s = np.abs(q.astype(np.float64)) @ np.repeat(np.abs(k.astype(np.float64)), g, 1).transpose(0, 1, 3, 2) / 8.0
+    if causal:
+        Tq, Tkv = s.shape[2:]
+        s[..., np.arange(Tkv)[None, :] > np.arange(Tq)[:, None] + Tkv - Tq] = 0.0
+    scores = s.max(-1, keepdims=True) * (2.0 ** -21 + 10 * 2.0 ** -24) + 2.0 ** -23
+    rel = 2.0 ** -21 + 2.0 ** -21 + (k.shape[2] // 64 + 12) * 2.0 ** -23
+    return np.all(np.abs(got - want) <= (2 * scores + rel) * size)
+
+
+@pytest.mark.parametrize("big", [1e6, 1e9, 1e12, 1e15, -1e17])
+@pytest.mark.parametrize("causal", [0, 1])
+def test_large_values_at_keys_that_do_not_count(causal, big):
+    """Keys that the mask removes, keys to come, and keys whose softmax weight is
+    nothing, with a V that is 10^6 .. 10^17 times the others': the outputs are
+    those of the keys that count."""
+    rng = np.random.default_rng(11)
+    q, k, v = data(rng, 2, 4, 2, 130, 200)
+    mask = np.zeros((130, 200), np.float32)
+    if causal:
+        v[:, :, 199] *= big            # seen by the last query only
+        v[0, :, 150, ::3] = big        # by some fifty of them
+        want = exact(q, k, v, 1)
+        got = gpu(q, k, v, 1)
+    else:
+        for fill in (-np.inf, np.finfo(np.float32).min, -1e30):
+            mask[:, 5] = mask[:, 70:72] = mask[3:, 199] = fill
+            v[:, :, 5] = v[:, :, 70:72] = big
+            v[0, :, 199, 1::2] = big
+            want, got = exact(q, k, v, 0, mask), gpu(q, k, v, 0, mask)
+            assert close(got, want, q, k, v, 0, mask)
+        # not masked: a score some 25 below the others', so 10^-11 of the weight
+        q[..., 0] = 40.0
+        k[..., 0] = 0.0
+        k[:, :, 33, 0] = -5.0
+        mask = None
+        v[:, :, 33] = big
+        want, got = exact(q, k, v, 0), gpu(q, k, v, 0)
+    assert close(got, want, q, k, v, causal, mask)
+
+
+@pytest.mark.parametrize("e", [8, 14, 20, 30])
+@pytest.mark.parametrize("Tq,Tkv", [(130, 200), (700, 700)])
+def test_units_of_dimensions(Tq, Tkv, e):
+    """Dimensions of q in units up to 2^e apart, those of k in the inverse ones;
+    columns of V with values 2^2e apart."""
+    rng = np.random.default_rng(13 + e)
+    q, k, v = data(rng, 1, 2, 1, Tq, Tkv)
+    f = rng.integers(-e, e + 1, (1, 1, 1, 64))
+    q, k = np.ldexp(q, f).astype(np.float32), np.ldexp(k, -f).astype(np.float32)
+    v = np.ldexp(v, rng.integers(-e, e + 1, v.shape)).astype(np.float32)
+    for causal in (0, 1):
+        assert close(gpu(q, k, v, causal), exact(q, k, v, causal), q, k, v, causal)
+
+
+def test_peaked_softmax():
+    """Scores of a wide range (weights from 1 down to nothing), queries and rows
+    of zeros, zero columns of V."""
+    rng = np.random.default_rng(17)
+    q, k, v = data(rng, 1, 2, 2, 300, 400)
+    q *= 12.0
+    q[0, 0, 7] = k[0, 1, 9] = 0.0
+    v[..., 5] = 0.0
+    v[0, 0, 100:, 6] = 0.0
+    for causal in (0, 1):
+        assert close(gpu(q, k, v, causal), exact(q, k, v, causal), q, k, v, causal)
