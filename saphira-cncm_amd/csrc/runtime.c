@@ -143,24 +143,34 @@ static size_t g_ws_size[WS_COUNT];
 static void *workspace(int slot, size_t bytes, int quiet) {
     if (bytes <= g_ws_size[slot]) return g_ws[slot];
     if (ncm_ready()) return NULL;
+    size_t sz = bytes < (1u << 20) ? (1u << 20) : bytes;
+    sz = (sz + 0xFFFFF) & ~(size_t)0xFFFFF;
+    void *p = NULL;
+    if (quiet) {
+        /* the new block first: where there is no room for it, the smaller calls
+         * keep the old one, with no wait and no allocation of theirs */
+        if (hipMalloc(&p, sz) != hipSuccess) {
+            (void)hipGetLastError();
+            return NULL;
+        }
+    }
     if (g_ws[slot]) {
         hipError_t e = hipStreamSynchronize(g_stream);
         if (e != hipSuccess) {
             if (!quiet) ncm_fail(NCM_E_HIP, "workspace grow sync: %s", hipGetErrorString(e));
+            if (p) (void)hipFree(p);
             return NULL;
         }
         (void)hipFree(g_ws[slot]);
         g_ws[slot] = NULL;
         g_ws_size[slot] = 0;
     }
-    size_t sz = bytes < (1u << 20) ? (1u << 20) : bytes;
-    sz = (sz + 0xFFFFF) & ~(size_t)0xFFFFF;
-    void *p = NULL;
-    hipError_t e = hipMalloc(&p, sz);
-    if (e != hipSuccess) {
-        if (quiet) (void)hipGetLastError();
-        else ncm_fail(NCM_E_OOM, "workspace of %zu bytes: %s", sz, hipGetErrorString(e));
-        return NULL;
+    if (!p) {
+        hipError_t e = hipMalloc(&p, sz);
+        if (e != hipSuccess) {
+            ncm_fail(NCM_E_OOM, "workspace of %zu bytes: %s", sz, hipGetErrorString(e));
+            return NULL;
+        }
     }
     g_ws[slot] = p;
     g_ws_size[slot] = sz;

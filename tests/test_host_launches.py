@@ -91,3 +91,17 @@ def test_capture_after_an_eager_call(host, name, args):
     assert not eager["error"] and not captured["error"] and launches(captured)
     assert not {"hipMalloc", "hipFree", "hipStreamSynchronize"} & set(captured["log"])
     assert not any(w.startswith(("split_", "vq_screen16", "vq_pack")) for w in captured["log"])
+
+
+def test_a_refused_workspace_leaves_the_smaller_one(host):
+    """Where the device has no room for a call's packed operands the call runs on
+    the FP32 kernels; calls that fit the workspace already held keep it, without
+    allocating, freeing or waiting."""
+    small, big = ("linear_fwd", (4096, 1024, 768)), ("linear_fwd", (16384, 3072, 768))
+    first, refused, again, grown = host([small, (*big, 0, 0, 24 << 20), small, big])
+    assert any(w.startswith("split_") for w in launches(first))
+    assert not refused["error"] and all(w.startswith("gemm_") for w in launches(refused))
+    assert not {"hipFree", "hipStreamSynchronize"} & set(refused["log"])
+    assert not {"hipMalloc", "hipFree", "hipStreamSynchronize"} & set(again["log"])
+    assert launches(again) == launches(first)
+    assert any(w.startswith("split_") for w in launches(grown))
