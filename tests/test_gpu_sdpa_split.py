@@ -108,7 +108,7 @@ def close(got, want, q, k, v, causal, mask=None):
     by sum |q k| / 8 times the 2^-21 of its pairs' representation (2 x 2^-23, l.l
     2^-22) and some ten roundings of the sums (10 x 2^-24), and by 2^-23 of the
     larger of 1 and the scores that the bound lets pass; p and V by as much of
-    themselves, their sum by 2^-20 and its roundings, one a tile."""
+    themselves, their sum by 2^-21 and its roundings, one a tile."""
     size = exact(q, k, np.abs(v), causal, mask)
     g = q.shape[1] // k.shape[1]
     s = np.abs(q.astype(np.float64)) @ np.repeat(np.abs(k.astype(np.float64)), g, 1).transpose(0, 1, 3, 2) / 8.0
@@ -116,7 +116,7 @@ def close(got, want, q, k, v, causal, mask=None):
         Tq, Tkv = s.shape[2:]
         s[..., np.arange(Tkv)[None, :] > np.arange(Tq)[:, None] + Tkv - Tq] = 0.0
     scores = s.max(-1, keepdims=True) * (2.0 ** -21 + 10 * 2.0 ** -24) + 2.0 ** -23
-    rel = 2.0 ** -21 + 2.0 ** -20 + (k.shape[2] // 64 + 12) * 2.0 ** -23
+    rel = 2.0 ** -21 + 2.0 ** -21 + (k.shape[2] // 64 + 12) * 2.0 ** -23
     return np.all(np.abs(got - want) <= (2 * scores + rel) * size)
 
 
