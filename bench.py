@@ -23,7 +23,8 @@ duration plus one event record -- and, for the split_* kernels (operands as
 fp16 pairs), plus the launch that packs both operands, which belongs to the
 call.  The roofline kernel is the one with the most time in such launches; its
 peak is the FP32 MFMA's, or for a split_* kernel a third of the FP16 MFMA's
-(three products per FP32 product).
+(three products per FP32 product).  "dtype" is that of the operands, results
+and sums; "operands" in the config says what the split_* kernels multiply.
 
 The CPU baseline runs the reference's own CPU code (oracle/_ref/libref.so,
 compiled from the reference sources) in a child process on a bounded sample
@@ -666,6 +667,8 @@ def main():
         "data": "synthetic",
         "config": {"workload": "BASELINE config 2: fp32 linear sweep, fwd + dX + dW + db, "
                                "M in {1,64,512,4096} x 5 (K->N) shapes",
+                   "operands": "fp32; split_* kernels hold each value as two fp16 numbers (23 of its 24 bits) and "
+                               "sum three fp16 products in fp32",
                    "calls_per_step": n, "gflop_per_step": round(total_flops / args.steps / 1e9, 3),
                    "frac_fp32_mfma_peak": round(value / PEAK_TFLOPS, 4),
                    "wall_s": round(wall, 4),
